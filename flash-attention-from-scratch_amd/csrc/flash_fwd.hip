@@ -170,7 +170,7 @@ struct Tile {
 // DMA plan of one wave for a K or V tile: DMA_ITERS 16-byte-per-lane buffer->LDS copies, each
 // filling 64 consecutive physical chunk slots of the swizzled tile; the lane reads the global
 // chunk whose swizzled home is its slot. Offsets are relative to the tile's first row.
-// KLAYOUT: the K-tile layout of the 16x16x32 path (fa::geom::m16_kslot_row / _chunk).
+// The 16x16x32 path's tiles are in fragment order (fa::geom::fo_*): KLAYOUT for a K tile.
 template <class T, bool KLAYOUT = false>
 struct TileDma {
     int voff[T::DMA_ITERS];  // byte offset of the lane's source chunk
@@ -182,12 +182,11 @@ struct TileDma {
             const int slot = slot0 + lane;
             int row = slot / T::CPR;
             int chunk;
-            if (KLAYOUT) {
-                row = g::m16_kslot_row(slot, T::D);
-                chunk = g::m16_kslot_chunk(slot, T::D);
+            if (T::M16) {
+                row = KLAYOUT ? g::fo_kslot_row(slot, T::D) : g::fo_vslot_row(slot, T::D);
+                chunk = KLAYOUT ? g::fo_kslot_chunk(slot, T::D) : g::fo_vslot_chunk(slot, T::D);
             } else {
-                chunk = T::M16 ? g::swizzle_chunk_m16(row, slot % T::CPR, T::D)
-                               : g::swizzle_chunk(row, slot % T::CPR, T::ROW_BYTES);
+                chunk = g::swizzle_chunk(row, slot % T::CPR, T::ROW_BYTES);
             }
             voff[it] = row * T::ROW_BYTES + 16 * chunk;
             lds0[it] = slot0 * 16;
@@ -919,8 +918,7 @@ __device__ __forceinline__ void end_phase() {
 // (lane % 16 and 16 + lane % 16) and keeps a running max and sum per query block. P^T of query
 // block qb and 32-key step t is the lane's own 8 exponentials, in the key order
 // fa::geom::pv16_key that the V^T operand reads. O^T in blocks oacc[db][qb] (features 16db..,
-// queries 16qb..). V tiles use the swizzle fa::geom::row_xor_m16; K tiles are stored so that
-// the K operand is read at the 32x32x16 path's conflict-free addresses (m16_kslot_row).
+// queries 16qb..). K and V tiles are stored in fragment order (fa::geom::fo_*).
 // Fragment reads and softmax VALU of the softmax phase, as "F, R, V": F of the 24 reads first,
 // then groups of {R reads, V VALU instructions} (R divides 24 - F). Non-causal tiles ask for
 // 16 reads before the first exponential and 8 per 24 VALU after; the compiler then issues all
@@ -1101,38 +1099,37 @@ struct M16 {
     static constexpr int DC = D / 32;      // 32-deep MFMA steps over D
     static constexpr int DB = D / 16;      // 16-wide feature blocks over D
     static constexpr int KS = T::BC / 32;  // 32-key steps of the P.V product
-    static constexpr int ROW = 2 * D;      // bytes per K/V row
     static constexpr int READS = KB * DC + 2 * KS * DB;
     static_assert(KB * QB * DC == 16 && DB * QB * KS == 16, "16 + 16 MFMAs per wave and tile");
 };
 
-// Lane-dependent LDS offsets: K fragment (kb, dc) at the 32x32x16 path's fragment address for
-// nb = kb / 2, kk = (kb % 2) * DC + dc (the K tile's own layout, fa::geom::m16_kslot_row);
-// V^T fragment db: the 4 rows pv16_key(lane, 0, 0..3) (via the tr16 addressing of a 4-row
-// block), 16 feature columns from 16db (the second read, keys pv16_key(lane, 0, 4..7), is 8
-// rows further; k step t is 32 rows further).
+// LDS reads of a tile in fragment order (fa::geom::fo_*): K operand (kb, dc) by one ds_read_b128,
+// V^T operand (t, db) by two ds_read_b64_tr_b16 (keys pv16_key(lane, t, 0..3) and 4..7). Three
+// lane offsets serve all 24 reads of a tile, whose distances are immediates. With row-major
+// tiles under XOR swizzles (the layout this replaced) every operand had a lane offset of its
+// own, 16 at d = 128: the ping-pong kernels now take 230-240 VGPRs (238-256 before) and the
+// d = 64 simple16 ones 116-117 (126-127). Interleaved A/B on MI355X, both layouts free of bank
+// conflicts: 16x16x1024 causal d = 128 93 -> 90 us, split-KV pass of 1x2x16384 causal 164.6 ->
+// 160.2 us, 4x16x3001 +0.6 %, 1x16x16384 +0.5 %, the d = 64 shapes -0.1 to +0.9 %.
 template <class T>
 struct Frag16 {
     using G = M16<T>;
-    int koff[G::KB][G::DC];
-    int voff[G::DB];
-    __device__ __forceinline__ explicit Frag16(int lane) {
-#pragma unroll
-        for (int kb = 0; kb < G::KB; ++kb)
-#pragma unroll
-            for (int dc = 0; dc < G::DC; ++dc)
-                koff[kb][dc] = g::tile_offset(32 * (kb >> 1) + (lane & 31),
-                                              2 * ((kb & 1) * G::DC + dc) + (lane >> 5), G::ROW);
-#pragma unroll
-        for (int db = 0; db < G::DB; ++db) {
-            const int row = g::pv16_key(lane, 0, 0) + g::tr16_row(lane);
-            const int c = 16 * db + g::tr16_col(lane);  // halves
-            voff[db] = g::tile_offset_m16(row, c >> 3, G::D) + 2 * (c & 7);
-        }
+    int k;     // K reads
+    int v[2];  // V^T reads of even and odd db
+    __device__ __forceinline__ explicit Frag16(int lane)
+        : k(g::fo_k_lane(lane)), v{g::fo_v_lane(lane), g::fo_v_lane(lane) ^ 32} {}
+    __device__ __forceinline__ f16x8 read_k(const char* kl, int kb, int dc) const {
+        return *reinterpret_cast<const f16x8*>(kl + k + g::fo_k_frag(kb, dc, G::D));
+    }
+    __device__ __forceinline__ f16x8 read_v(const char* vl, int t, int db) const {
+        const char* base = vl + v[db & 1];
+        const f16x4 lo = lds_read_tr16(base + g::fo_v_frag(t, db, 0, G::D));
+        const f16x4 up = lds_read_tr16(base + g::fo_v_frag(t, db, 1, G::D));
+        return f16x8{lo[0], lo[1], lo[2], lo[3], up[0], up[1], up[2], up[3]};
     }
 };
 
-// Q^T operands: qf[qb][dc] holds Q[qw + 16qb + lane%16][8 * m16_kchunk(dc, lane/16) .. +7],
+// Q^T operands: qf[qb][dc] holds Q[qw + 16qb + lane%16][8 * fo_kchunk(dc, lane/16) .. +7],
 // the feature order of the K operand.
 template <class T>
 __device__ __forceinline__ void load_q16(const f16* qh, int qw, int n, int lane, int negate_q,
@@ -1144,8 +1141,7 @@ __device__ __forceinline__ void load_q16(const f16* qh, int qw, int n, int lane,
         const f16* src = qh + static_cast<size_t>(row) * G::D;
 #pragma unroll
         for (int dc = 0; dc < G::DC; ++dc) {
-            qf[qb][dc] =
-                *reinterpret_cast<const f16x8*>(src + 8 * g::m16_kchunk(dc, lane >> 4, G::D));
+            qf[qb][dc] = *reinterpret_cast<const f16x8*>(src + 8 * g::fo_kchunk(dc, lane >> 4));
             if (negate_q) qf[qb][dc] = -qf[qb][dc];
         }
     }
@@ -1161,7 +1157,7 @@ __device__ __forceinline__ void load_k16(const char* kl, const Frag16<T>& fr,
     for (int kb = 0; kb < G::KB; ++kb)
 #pragma unroll
         for (int dc = 0; dc < G::DC; ++dc)
-            kf[kb][dc] = *reinterpret_cast<const f16x8*>(kl + fr.koff[kb][dc]);
+            kf[kb][dc] = fr.read_k(kl, kb, dc);
 }
 template <class T>
 __device__ __forceinline__ void load_v16(const char* vl, const Frag16<T>& fr,
@@ -1170,12 +1166,7 @@ __device__ __forceinline__ void load_v16(const char* vl, const Frag16<T>& fr,
 #pragma unroll
     for (int t = 0; t < G::KS; ++t)
 #pragma unroll
-        for (int db = 0; db < G::DB; ++db) {
-            const char* base = vl + fr.voff[db] + 32 * t * G::ROW;
-            const f16x4 lo = lds_read_tr16(base);
-            const f16x4 up = lds_read_tr16(base + 8 * G::ROW);
-            vf[t][db] = f16x8{lo[0], lo[1], lo[2], lo[3], up[0], up[1], up[2], up[3]};
-        }
+        for (int db = 0; db < G::DB; ++db) vf[t][db] = fr.read_v(vl, t, db);
 }
 
 // S^T = K Q^T of one tile (the first one, before the steady phases).
@@ -1659,8 +1650,8 @@ __global__ __launch_bounds__(T::THREADS) void flash_fwd_pingpong16(
     using I1 = std::integral_constant<int, 1>;
     using I2 = std::integral_constant<int, 2>;
 
-    const TileDma<T, true> dma_k(wave, lane);  // K tiles in the layout of Frag16's K reads
-    const TileDma<T> dma(wave, lane);          // V tiles, swizzle fa::geom::row_xor_m16
+    const TileDma<T, true> dma_k(wave, lane);  // K tiles, fragment order
+    const TileDma<T> dma(wave, lane);          // V tiles, fragment order
     f16x8 qf[G::QB][G::DC];
     float m_run[G::QB] = {-INFINITY, -INFINITY};
     if constexpr (FAST) {
@@ -2044,8 +2035,7 @@ __device__ __forceinline__ void qk16_lean(const char* kl, const Frag16<T>& fr,
     for (int kb = 0; kb < G::KB; ++kb) {
         f16x8 kf[G::DC];
 #pragma unroll
-        for (int dc = 0; dc < G::DC; ++dc)
-            kf[dc] = *reinterpret_cast<const f16x8*>(kl + fr.koff[kb][dc]);
+        for (int dc = 0; dc < G::DC; ++dc) kf[dc] = fr.read_k(kl, kb, dc);
 #pragma unroll
         for (int qb = 0; qb < G::QB; ++qb) {
             s[kb][qb] = f32x4{};
@@ -2065,12 +2055,7 @@ __device__ __forceinline__ void pv16_lean(const char* vl, const Frag16<T>& fr,
     for (int t = 0; t < G::KS; ++t) {
         f16x8 vf[G::DB];
 #pragma unroll
-        for (int db = 0; db < G::DB; ++db) {
-            const char* base = vl + fr.voff[db] + 32 * t * G::ROW;
-            const f16x4 lo = lds_read_tr16(base);
-            const f16x4 up = lds_read_tr16(base + 8 * G::ROW);
-            vf[db] = f16x8{lo[0], lo[1], lo[2], lo[3], up[0], up[1], up[2], up[3]};
-        }
+        for (int db = 0; db < G::DB; ++db) vf[db] = fr.read_v(vl, t, db);
 #pragma unroll
         for (int db = 0; db < G::DB; ++db)
 #pragma unroll
@@ -2184,8 +2169,7 @@ __device__ __forceinline__ void softmax16_any(const f32x4 (&s)[M16<T>::KB][M16<T
 
 // flash_fwd_kernel's schedule (per tile: barrier, prefetch, then S = QK^T, mask, softmax and
 // O += PV in turn; the item's first tile peeled off) on the ping-pong's 16x16x32 MFMAs and
-// layouts (K tiles in the Frag16 read layout, V tiles with row_xor_m16, P^T straight from the
-// lane's own exponentials). Each wave holds 32 query rows as two 16-row blocks, and each lane
+// layouts (K and V tiles in fragment order, P^T straight from the lane's own exponentials). Each wave holds 32 query rows as two 16-row blocks, and each lane
 // 4 keys of 2 queries per 16-key block. Same arguments, grid and results as flash_fwd_kernel.
 template <class T, bool CAUSAL, bool SPLIT = false>
 __global__ __launch_bounds__(T::THREADS) void flash_fwd_simple16(
@@ -2235,8 +2219,8 @@ __global__ __launch_bounds__(T::THREADS) void flash_fwd_simple16(
     };
 
     constexpr int PRIO = T::D == 128 ? FA_SIMPLE_PRIO_D128 : FA_SIMPLE_PRIO_D64;
-    const TileDma<T, true> dma_k(wave, lane);  // K tiles in the layout of Frag16's K reads
-    const TileDma<T> dma(wave, lane);          // V tiles, swizzle fa::geom::row_xor_m16
+    const TileDma<T, true> dma_k(wave, lane);  // K tiles, fragment order
+    const TileDma<T> dma(wave, lane);          // V tiles, fragment order
     load_tile<T>(kh, j_begin * T::BC, n, kbuf(I0{}), dma_k);
     load_tile<T>(vh, j_begin * T::BC, n, vbuf(I0{}), dma);
     if constexpr (NBUF == 3) {

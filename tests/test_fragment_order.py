@@ -1,0 +1,74 @@
+"""CPU: the fragment-order LDS tiles of the 16x16x32 kernels (fa::geom::fo_*).
+
+The DMA's slot maps and the kernels' read addresses must give every lane the MFMA operand it
+needs, from the geometry alone: each 16-byte slot holds one cell of the tile, a K read returns
+key row m16_key(kb, lane % 16) and chunk fo_kchunk(dc, lane / 16), a V^T read the four keys and
+four columns that ds_read_b64_tr_b16 expects of the lane; no read has a bank conflict in the lane
+groups the hardware serves at once; and four consecutive lanes of a DMA request read 64
+contiguous bytes.
+"""
+
+from __future__ import annotations
+
+import pytest
+
+from test_geometry import geo  # noqa: F401  (the host build of fa_geometry.h)
+
+DIMS = [64, 128]
+# lanes a ds_read_b128 serves together (measured on MI355X)
+B128_GROUPS = [[*range(0, 4), *range(12, 16), *range(20, 28)],
+               [*range(4, 12), *range(16, 20), *range(28, 32)]]
+B128_GROUPS += [[lane + 32 for lane in grp] for grp in B128_GROUPS]
+
+
+def _cells(geo, d):  # noqa: F811
+    k = [(geo.geom_fo_kslot_row(s, d), geo.geom_fo_kslot_chunk(s, d)) for s in range(512)]
+    v = [(geo.geom_fo_vslot_row(s, d), geo.geom_fo_vslot_chunk(s, d)) for s in range(512)]
+    return k, v
+
+
+@pytest.mark.parametrize("d", DIMS)
+def test_slots_hold_every_cell_once_and_requests_read_64_byte_pieces(geo, d):  # noqa: F811
+    want = {(r, c) for r in range(4096 // d) for c in range(d // 8)}
+    for cells in _cells(geo, d):
+        assert set(cells) == want and len(cells) == len(want)
+        for s in range(0, 512, 4):
+            rows, chunks = zip(*cells[s:s + 4])
+            assert len(set(rows)) == 1 and min(chunks) % 4 == 0
+            assert sorted(chunks) == list(range(min(chunks), min(chunks) + 4))
+
+
+@pytest.mark.parametrize("d", DIMS)
+def test_k_reads_get_the_operand_without_conflicts(geo, d):  # noqa: F811
+    cells, _ = _cells(geo, d)
+    lanes = [geo.geom_fo_k_lane(lane) for lane in range(64)]
+    for kb in range(4096 // d // 16):
+        for dc in range(d // 32):
+            off = geo.geom_fo_k_frag(kb, dc, d)
+            for lane in range(64):
+                assert (lanes[lane] + off) % 16 == 0
+                assert cells[(lanes[lane] + off) // 16] == (geo.geom_m16_key(kb, lane % 16),
+                                                            geo.geom_fo_kchunk(dc, lane // 16))
+    assert sorted(geo.geom_fo_kchunk(dc, grp) for dc in range(d // 32) for grp in range(4)) == \
+        list(range(d // 8))
+    for grp in B128_GROUPS:
+        assert sorted(lanes[lane] % 256 // 16 for lane in grp) == list(range(16))
+        assert sum(lanes[lane] >= 4096 for lane in grp) == 8
+
+
+@pytest.mark.parametrize("d", DIMS)
+def test_v_reads_get_the_operand_without_conflicts(geo, d):  # noqa: F811
+    _, cells = _cells(geo, d)
+    for t in range(4096 // d // 32):
+        for db in range(d // 16):
+            for e in range(2):
+                addr = [(geo.geom_fo_v_lane(lane) ^ (32 * (db % 2))) +
+                        geo.geom_fo_v_frag(t, db, e, d) for lane in range(64)]
+                for lane, a in enumerate(addr):
+                    row, chunk = cells[a // 16]
+                    col = 8 * chunk + a % 16 // 2
+                    first = geo.geom_pv16_key(lane, t, 4 * e)  # keys first..first + 3
+                    assert row == first + geo.geom_tr16_row(lane)
+                    assert col == 16 * db + geo.geom_tr16_col(lane)
+                for half in (addr[:32], addr[32:]):
+                    assert sorted(a % 256 // 8 for a in half) == list(range(32))
