@@ -326,6 +326,15 @@ constexpr Work work_of_xcd(int block_id, int bh_count, int n_qblocks, bool causa
     return Work{static_cast<int>(t / n_qblocks), static_cast<int>(t % n_qblocks)};
 }
 
+// Causal grids of 257 to 512 workgroups that are all resident at once, two per CU (the two-way
+// key split): the workgroups after the first 256 take their blocks shortest first, so that the CU
+// that got the longest block also gets the shortest. Measured on MI355X against the plain
+// longest-first order: 1x40x700 d = 128 14.7 -> 14.1 us, 2x16x900 16.4 -> 15.9, 1x32x1000 18.1 ->
+// 17.8, 1x16x2000 28.3 -> 27.9 (other grids keep the order).
+constexpr int two_round_turn(int block_id, int total) {
+    return total > 256 && total <= 512 && block_id >= 256 ? total + 255 - block_id : block_id;
+}
+
 // Causal grids of paired query blocks: workgroup id -> (batch*head index, long query block
 // n_qblocks - 1 - p, short query block p, or -1 when p is the middle block of an odd count).
 // A causal query block qb visits qb + 1 key blocks, so every pair visits n_qblocks + 1 and all

@@ -136,7 +136,7 @@ static_assert(FA_SIMPLE_NBUF == 2 || FA_SIMPLE_NBUF == 3, "two or three K/V buff
 #define FA_SIMPLE_PRIO_D128 1
 #endif
 
-template <int D_, int BC_, int NW_, bool LAZY_, int SCHED_>
+template <int D_, int BC_, int NW_, bool LAZY_, int SCHED_, bool M16_ = SCHED_ != SIMPLE>
 struct Tile {
     static constexpr int D = D_;            // head dim (64 or 128)
     static constexpr int BC = BC_;          // keys per K/V tile
@@ -150,7 +150,7 @@ struct Tile {
     static constexpr int ROW_BYTES = 2 * D;
     static constexpr int CPR = D / 8;                  // 16-byte chunks per row
     static constexpr int TILE_BYTES = BC * ROW_BYTES;  // one K or V tile
-    static constexpr bool M16 = SCHED == PINGPONG16 || SCHED == SIMPLE16;  // 16x16x32 layouts
+    static constexpr bool M16 = M16_;                  // 16x16x32 MFMAs and layouts
     static constexpr int NBUF =  // per K, V (the simple schedule's third only within 64 KiB)
         SCHED == PINGPONG16 ? 3
                             : ((SCHED == SIMPLE || SCHED == SIMPLE16) && 6 * TILE_BYTES <= 64 * 1024
@@ -647,213 +647,6 @@ __global__ __launch_bounds__(256) void flash_fwd_combine(
     if (lse != nullptr && c == 0) lse[row] = (m + __builtin_amdgcn_logf(wsum)) * kLn2;
 }
 
-// ---- kernel, key-split schedule (small grids) --------------------------------------------------
-// KS waves per 32 query rows (KS = 2, or 4 for grids of one workgroup per CU): wave w takes key
-// tiles part, part + KS, part + 2 KS, ... of the query block (part = w / NW), each with its own
-// running max, row sum and O (simple schedule per tile). At the end the parts merge pairwise
-// through LDS in log2(KS) rounds, part p + d handing (m, l, O) to part p (d = KS/2, ..., 1),
-// which merges them (O = 2^(m_a - m) O_a + 2^(m_b - m) O_b, l likewise); part 0 stores. KS times
-// the waves of the simple schedule on the same grid, for grids too small to fill the GPU, with
-// no workspace.
-template <class T, bool CAUSAL>
-__global__ __launch_bounds__(T::THREADS) void flash_fwd_ksplit(
-    const f16* __restrict__ q, const f16* __restrict__ k, const f16* __restrict__ v,
-    f16* __restrict__ o, float* __restrict__ lse, int n, int bh_count, int n_qblocks,
-    float scale_log2, int negate_q, int /*tiles_per_split*/, float* /*o_part*/,
-    float* /*lse_part*/, unsigned /*launch_id*/, int group_heads) {
-    constexpr int KS = T::KS;
-    static_assert(KS == 2 || KS == 4, "two or four key parts");
-    // One LDS object per (key part, buffer) for K and V, and the buffer of each step fixed at
-    // compile time (the step loop is unrolled by two): the compiler then sees that a refill
-    // cannot alias the reads of the other buffer and waits for DMA only at the step barrier.
-    // (Parts 2 and 3 exist only with KS = 4.) The merge reuses buffer 0 of each part.
-    __shared__ __attribute__((aligned(1024))) char k00[T::TILE_BYTES];
-    __shared__ __attribute__((aligned(1024))) char k01[T::TILE_BYTES];
-    __shared__ __attribute__((aligned(1024))) char k10[T::TILE_BYTES];
-    __shared__ __attribute__((aligned(1024))) char k11[T::TILE_BYTES];
-    __shared__ __attribute__((aligned(1024))) char k20[T::TILE_BYTES];
-    __shared__ __attribute__((aligned(1024))) char k21[T::TILE_BYTES];
-    __shared__ __attribute__((aligned(1024))) char k30[T::TILE_BYTES];
-    __shared__ __attribute__((aligned(1024))) char k31[T::TILE_BYTES];
-    __shared__ __attribute__((aligned(1024))) char v00[T::TILE_BYTES];
-    __shared__ __attribute__((aligned(1024))) char v01[T::TILE_BYTES];
-    __shared__ __attribute__((aligned(1024))) char v10[T::TILE_BYTES];
-    __shared__ __attribute__((aligned(1024))) char v11[T::TILE_BYTES];
-    __shared__ __attribute__((aligned(1024))) char v20[T::TILE_BYTES];
-    __shared__ __attribute__((aligned(1024))) char v21[T::TILE_BYTES];
-    __shared__ __attribute__((aligned(1024))) char v30[T::TILE_BYTES];
-    __shared__ __attribute__((aligned(1024))) char v31[T::TILE_BYTES];
-    static_assert(T::NW * 64 * 8 <= T::TILE_BYTES && T::NW * 64 * 16 * 4 <= T::TILE_BYTES,
-                  "the merge's (m, l) and O blocks fit in one tile buffer each");
-
-    const int lane = threadIdx.x & 63;
-    const int wave = wave_uniform(threadIdx.x >> 6);
-    const int part = wave / T::NW;  // key tiles part, part + KS, ...
-    const int wq = wave % T::NW;    // which 32 query rows
-    const g::Work w = g::work_of_xcd(blockIdx.x, bh_count, n_qblocks, CAUSAL, group_heads);
-    const size_t head = static_cast<size_t>(w.bh) * n * T::D;
-    const f16* kh = k + head;
-    const f16* vh = v + head;
-    const int q0 = w.qb * T::BR;
-    const int qw = q0 + wq * 32;
-    const int qrow = qw + (lane & 31);
-    const int n_tiles = g::num_kv_tiles(n, q0, T::BR, T::BC, CAUSAL);
-    const int n_steps = (n_tiles + KS - 1) / KS;
-    using I0 = std::integral_constant<int, 0>;
-    using I1 = std::integral_constant<int, 1>;
-    // Buffer b of key part H (both compile-time).
-    auto kbuf = [&](auto hc, auto b) {
-        constexpr int H = decltype(hc)::value;
-        constexpr int B = decltype(b)::value;
-        if constexpr (H == 0) return B == 0 ? k00 : k01;
-        else if constexpr (H == 1) return B == 0 ? k10 : k11;
-        else if constexpr (H == 2) return B == 0 ? k20 : k21;
-        else return B == 0 ? k30 : k31;
-    };
-    auto vbuf = [&](auto hc, auto b) {
-        constexpr int H = decltype(hc)::value;
-        constexpr int B = decltype(b)::value;
-        if constexpr (H == 0) return B == 0 ? v00 : v01;
-        else if constexpr (H == 1) return B == 0 ? v10 : v11;
-        else if constexpr (H == 2) return B == 0 ? v20 : v21;
-        else return B == 0 ? v30 : v31;
-    };
-    // Calls f with the wave's part as a compile-time constant (wave-uniform branch).
-    auto with_part = [&](auto&& f) {
-        if constexpr (KS == 4) {
-            if (part == 3) return f(std::integral_constant<int, 3>{});
-            if (part == 2) return f(std::integral_constant<int, 2>{});
-        }
-        if (part == 1) return f(I1{});
-        return f(I0{});
-    };
-
-    const TileDma<T> dma(wq, lane);
-    with_part([&](auto hc) {
-        constexpr int H = decltype(hc)::value;
-        if (H < n_tiles) {
-            load_tile<T>(kh, H * T::BC, n, kbuf(hc, I0{}), dma);
-            load_tile<T>(vh, H * T::BC, n, vbuf(hc, I0{}), dma);
-        }
-    });
-    f16x8 qf[T::KK];
-    load_q<T>(q + head, qrow, n, lane, negate_q, qf);
-    const Frag<T> fr(lane);
-
-    f32x16 oacc[T::DB];
-#pragma unroll
-    for (int db = 0; db < T::DB; ++db) oacc[db] = f32x16{};
-    float m_run = -INFINITY;
-    float l_run = 0.0F;
-
-    // Step j in buffer B = j % 2: key part H's tile KS j + H.
-    auto step = [&](int j, auto hc, auto b, auto first) {
-        constexpr int H = decltype(hc)::value;
-        using Other = std::integral_constant<int, 1 - decltype(b)::value>;
-        wait_vmem();
-        __syncthreads();  // step j's tiles are in LDS; step j-1's buffers are free
-        const int tn = KS * (j + 1) + H;
-        if (tn < n_tiles) {
-            load_tile<T>(kh, tn * T::BC, n, kbuf(hc, Other{}), dma);
-            load_tile<T>(vh, tn * T::BC, n, vbuf(hc, Other{}), dma);
-        }
-        const int t = KS * j + H;
-        const int kt = t * T::BC;
-        if (t >= n_tiles || qw >= n || g::tile_fully_masked(kt, qw, 32, CAUSAL)) return;
-        f32x16 s[T::NB];
-        qk_tile<T>(kbuf(hc, b), fr, qf, s);
-        if (g::tile_needs_mask(n, kt, T::BC, qw, CAUSAL)) mask_tile<T, CAUSAL>(s, kt, n, qrow, lane);
-        f16x8 p[T::NB][2];
-        softmax_any<T, decltype(first)::value>(s, scale_log2, m_run, l_run, oacc, p);
-        pv_tile<T>(vbuf(hc, b), fr, p, oacc);
-    };
-    // wave-uniform branch; every part passes the same number of barriers. n_steps >= 1; step 0
-    // (each part's first tile) is peeled off.
-    with_part([&](auto hc) {
-        using Later = std::false_type;
-        step(0, hc, I0{}, std::true_type{});
-        int j = 1;
-        for (; j + 2 <= n_steps; j += 2) {
-            step(j, hc, I1{}, Later{});
-            step(j + 1, hc, I0{}, Later{});
-        }
-        if (j < n_steps) step(j, hc, I1{}, Later{});
-    });
-
-    // Merge. In round d (d = KS/2, ..., 1), part p + d (p < d) writes (m, l) to its buffer k_0
-    // and then O, one 32-column block at a time, to its buffer v_0; part p merges. Lanes write
-    // 8 and 16 bytes at consecutive addresses (O as four 16-byte pieces per block, piece-major),
-    // which keeps every access free of bank conflicts.
-    float l_tot = sum_xor32(l_run);
-    const int slot = wq * 64 + lane;
-    wait_vmem();
-    __syncthreads();  // every wave is done with the tile buffers
-#pragma unroll
-    for (int d = KS / 2; d >= 1; d /= 2) {
-        const bool sender = part >= d && part < 2 * d;
-        const bool receiver = part < d;
-        // buffers k_0 and v_0 of part src (1, 2 or 3: a sender), read by its receiver too
-        auto ml_of = [&](int src) -> float* {
-            if constexpr (KS == 4) {
-                if (src == 3) return reinterpret_cast<float*>(k30);
-                if (src == 2) return reinterpret_cast<float*>(k20);
-            }
-            return reinterpret_cast<float*>(k10);
-        };
-        auto ob_of = [&](int src) -> float* {
-            if constexpr (KS == 4) {
-                if (src == 3) return reinterpret_cast<float*>(v30);
-                if (src == 2) return reinterpret_cast<float*>(v20);
-            }
-            return reinterpret_cast<float*>(v10);
-        };
-        if (sender) {
-            *reinterpret_cast<f32x2*>(ml_of(part) + 2 * slot) = f32x2{m_run, l_tot};
-        }
-        __syncthreads();
-        float wa = 1.0F, wb = 0.0F;
-        if (receiver) {
-            const f32x2 mb_lb = *reinterpret_cast<const f32x2*>(ml_of(part + d) + 2 * slot);
-            const float mb = mb_lb[0];
-            const float m_new = fmaxf(m_run, mb);
-            // a part that saw no key has m = -inf and weighs 0; both -inf only for rows >= n
-            wa = m_run == -INFINITY ? 0.0F : exp2_fast(m_run - m_new);
-            wb = mb == -INFINITY ? 0.0F : exp2_fast(mb - m_new);
-            l_tot = l_tot * wa + mb_lb[1] * wb;
-            m_run = m_new;
-        }
-#pragma unroll
-        for (int db = 0; db < T::DB; ++db) {
-            if (sender) {
-                float* ob = ob_of(part);
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    *reinterpret_cast<f32x4*>(ob + 4 * (r * T::NW * 64 + slot)) =
-                        f32x4{oacc[db][4 * r], oacc[db][4 * r + 1], oacc[db][4 * r + 2],
-                              oacc[db][4 * r + 3]};
-                }
-            }
-            __syncthreads();
-            if (receiver) {
-                const float* ob = ob_of(part + d);
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const f32x4 x = *reinterpret_cast<const f32x4*>(ob + 4 * (r * T::NW * 64 + slot));
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) {
-                        oacc[db][4 * r + i] = oacc[db][4 * r + i] * wa + x[i] * wb;
-                    }
-                }
-            }
-            __syncthreads();
-        }
-    }
-    if (part == 0) {
-        store_o_tot<T>(o + head, lse ? lse + static_cast<size_t>(w.bh) * n : nullptr, qrow, n,
-                       lane, m_run, l_tot, oacc);
-    }
-}
-
 // ---- ping-pong schedule: phase protocol ---------------------------------------------------------
 // Eight waves, two groups of four: the hardware deals the waves of a workgroup round-robin to
 // the four SIMDs of the CU, so waves w and w+4 share a SIMD. Every wave alternates two phases
@@ -1116,8 +909,10 @@ struct Frag16 {
     using G = M16<T>;
     int k;     // K reads
     int v[2];  // V^T reads of even and odd db
-    __device__ __forceinline__ explicit Frag16(int lane)
-        : k(g::fo_k_lane(lane)), v{g::fo_v_lane(lane), g::fo_v_lane(lane) ^ 32} {}
+    // base: byte offset of the tile in its LDS buffer
+    __device__ __forceinline__ explicit Frag16(int lane, int base = 0)
+        : k(g::fo_k_lane(lane) + base),
+          v{g::fo_v_lane(lane) + base, (g::fo_v_lane(lane) ^ 32) + base} {}
     __device__ __forceinline__ f16x8 read_k(const char* kl, int kb, int dc) const {
         return *reinterpret_cast<const f16x8*>(kl + k + g::fo_k_frag(kb, dc, G::D));
     }
@@ -1351,6 +1146,51 @@ __device__ __forceinline__ void softmax16_tile(const f32x4 (&s)[M16<T>::KB][M16<
         }
         // without ADD_SUM the caller adds the row sums of p (matrix_phase16<T, true>)
         l_run[qb] = (rescale ? l_run[qb] * alpha[qb] : l_run[qb]) + sum;
+    }
+}
+
+// Row sums of P on the matrix cores: A = ones, so that every lane of a query receives the sum over
+// the step's 32 keys (all four accumulators alike, no reduction across lanes left).
+template <class T>
+__device__ __forceinline__ f32x4 rowsum16(const f16x8 (&p)[M16<T>::KS], f32x4 l) {
+    const f16 o = static_cast<f16>(1.0F);
+    const f16x8 ones = {o, o, o, o, o, o, o, o};
+#pragma unroll
+    for (int t = 0; t < M16<T>::KS; ++t) l = mfma16(ones, p[t], l);
+    return l;
+}
+
+// softmax16_optimistic / softmax16_tile with the row sums on the matrix cores (l: rowsum16).
+template <class T>
+__device__ __forceinline__ void softmax16_optimistic_mx(
+    const f32x4 (&s)[M16<T>::KB][M16<T>::QB], float scale_log2, const float (&m_run)[M16<T>::QB],
+    f32x4 (&l)[M16<T>::QB], bool& overflow, f16x8 (&p)[M16<T>::QB][M16<T>::KS]) {
+    using G = M16<T>;
+    softmax16_unchecked<T>(s, scale_log2, m_run, p);
+    f32x4 ln[G::QB];
+    bool bad = false;
+#pragma unroll
+    for (int qb = 0; qb < G::QB; ++qb) {
+        ln[qb] = rowsum16<T>(p[qb], l[qb]);
+        bad = bad || !(ln[qb][0] < INFINITY);
+    }
+    overflow = wave_any(bad);
+#pragma unroll
+    for (int qb = 0; qb < G::QB; ++qb) l[qb] = overflow ? l[qb] : ln[qb];
+}
+template <class T>
+__device__ __forceinline__ void softmax16_tile_mx(const f32x4 (&s)[M16<T>::KB][M16<T>::QB],
+                                                  float scale_log2, float (&m_run)[M16<T>::QB],
+                                                  f32x4 (&l)[M16<T>::QB],
+                                                  float (&alpha)[M16<T>::QB], bool& rescale,
+                                                  f16x8 (&p)[M16<T>::QB][M16<T>::KS]) {
+    using G = M16<T>;
+    float unused[G::QB] = {0.0F, 0.0F};
+    softmax16_tile<T, false>(s, scale_log2, m_run, unused, alpha, rescale, p);
+#pragma unroll
+    for (int qb = 0; qb < G::QB; ++qb) {
+        if (rescale) l[qb] *= alpha[qb];
+        l[qb] = rowsum16<T>(p[qb], l[qb]);
     }
 }
 
@@ -2309,6 +2149,587 @@ __global__ __launch_bounds__(T::THREADS) void flash_fwd_simple16(
                    : g::work_of_xcd(blockIdx.x, bh_count, n_qblocks, CAUSAL, group_heads));
 }
 
+// ---- kernel, key-split schedule on 32x32x16 MFMAs (short rows) ----------------------------------
+// Two waves per 32 query rows: wave w takes key tiles part, part + 2, ... of the query block
+// (part = w / NW), each with its own running max, row sum and O (simple schedule per tile); at the
+// end part 1 hands (m, l, O) to part 0 through LDS, which merges them (O = 2^(m_a - m) O_a +
+// 2^(m_b - m) O_b, l likewise) and stores. Kept for short rows (FA_KS_SHORT_*), where a launch is a
+// few steps between its fixed costs: the 16x16x32 key split, whose lanes hold two queries, has more
+// instructions in its first softmax and its merge, and requests past a block's last tile.
+template <class T, bool CAUSAL>
+__global__ __launch_bounds__(T::THREADS) void flash_fwd_ksplit(
+    const f16* __restrict__ q, const f16* __restrict__ k, const f16* __restrict__ v,
+    f16* __restrict__ o, float* __restrict__ lse, int n, int bh_count, int n_qblocks,
+    float scale_log2, int negate_q, int /*tiles_per_split*/, float* /*o_part*/,
+    float* /*lse_part*/, unsigned /*launch_id*/, int group_heads) {
+    constexpr int KS = T::KS;
+    static_assert(KS == 2 && !T::M16, "two key parts on 32x32x16 MFMAs");
+    // One LDS object per (key part, buffer) for K and V, and the buffer of each step fixed at
+    // compile time (the step loop is unrolled by two): the compiler then sees that a refill
+    // cannot alias the reads of the other buffer and waits for DMA only at the step barrier.
+    // The merge reuses buffer 0 of part 1.
+    __shared__ __attribute__((aligned(1024))) char k00[T::TILE_BYTES];
+    __shared__ __attribute__((aligned(1024))) char k01[T::TILE_BYTES];
+    __shared__ __attribute__((aligned(1024))) char k10[T::TILE_BYTES];
+    __shared__ __attribute__((aligned(1024))) char k11[T::TILE_BYTES];
+    __shared__ __attribute__((aligned(1024))) char v00[T::TILE_BYTES];
+    __shared__ __attribute__((aligned(1024))) char v01[T::TILE_BYTES];
+    __shared__ __attribute__((aligned(1024))) char v10[T::TILE_BYTES];
+    __shared__ __attribute__((aligned(1024))) char v11[T::TILE_BYTES];
+    static_assert(T::NW * 64 * 8 <= T::TILE_BYTES && T::NW * 64 * 16 * 4 <= T::TILE_BYTES,
+                  "the merge's (m, l) and O blocks fit in one tile buffer each");
+
+    const int lane = threadIdx.x & 63;
+    const int wave = wave_uniform(threadIdx.x >> 6);
+    const int part = wave / T::NW;  // key tiles part, part + KS, ...
+    const int wq = wave % T::NW;    // which 32 query rows
+    const g::Work w = g::work_of_xcd(blockIdx.x, bh_count, n_qblocks, CAUSAL, group_heads);
+    const size_t head = static_cast<size_t>(w.bh) * n * T::D;
+    const f16* kh = k + head;
+    const f16* vh = v + head;
+    const int q0 = w.qb * T::BR;
+    const int qw = q0 + wq * 32;
+    const int qrow = qw + (lane & 31);
+    const int n_tiles = g::num_kv_tiles(n, q0, T::BR, T::BC, CAUSAL);
+    const int n_steps = (n_tiles + KS - 1) / KS;
+    using I0 = std::integral_constant<int, 0>;
+    using I1 = std::integral_constant<int, 1>;
+    // Buffer b of key part H (both compile-time).
+    auto kbuf = [&](auto hc, auto b) {
+        constexpr int H = decltype(hc)::value;
+        constexpr int B = decltype(b)::value;
+        if constexpr (H == 0) return B == 0 ? k00 : k01;
+        else return B == 0 ? k10 : k11;
+    };
+    auto vbuf = [&](auto hc, auto b) {
+        constexpr int H = decltype(hc)::value;
+        constexpr int B = decltype(b)::value;
+        if constexpr (H == 0) return B == 0 ? v00 : v01;
+        else return B == 0 ? v10 : v11;
+    };
+    // Calls f with the wave's part as a compile-time constant (wave-uniform branch).
+    auto with_part = [&](auto&& f) {
+        if (part == 1) return f(I1{});
+        return f(I0{});
+    };
+
+    const TileDma<T> dma(wq, lane);
+    with_part([&](auto hc) {
+        constexpr int H = decltype(hc)::value;
+        if (H < n_tiles) {
+            load_tile<T>(kh, H * T::BC, n, kbuf(hc, I0{}), dma);
+            load_tile<T>(vh, H * T::BC, n, vbuf(hc, I0{}), dma);
+        }
+    });
+    f16x8 qf[T::KK];
+    load_q<T>(q + head, qrow, n, lane, negate_q, qf);
+    const Frag<T> fr(lane);
+
+    f32x16 oacc[T::DB];
+#pragma unroll
+    for (int db = 0; db < T::DB; ++db) oacc[db] = f32x16{};
+    float m_run = -INFINITY;
+    float l_run = 0.0F;
+
+    // Step j in buffer B = j % 2: key part H's tile KS j + H.
+    auto step = [&](int j, auto hc, auto b, auto first) {
+        constexpr int H = decltype(hc)::value;
+        using Other = std::integral_constant<int, 1 - decltype(b)::value>;
+        wait_vmem();
+        __syncthreads();  // step j's tiles are in LDS; step j-1's buffers are free
+        const int tn = KS * (j + 1) + H;
+        if (tn < n_tiles) {
+            load_tile<T>(kh, tn * T::BC, n, kbuf(hc, Other{}), dma);
+            load_tile<T>(vh, tn * T::BC, n, vbuf(hc, Other{}), dma);
+        }
+        const int t = KS * j + H;
+        const int kt = t * T::BC;
+        if (t >= n_tiles || qw >= n || g::tile_fully_masked(kt, qw, 32, CAUSAL)) return;
+        f32x16 s[T::NB];
+        qk_tile<T>(kbuf(hc, b), fr, qf, s);
+        if (g::tile_needs_mask(n, kt, T::BC, qw, CAUSAL)) mask_tile<T, CAUSAL>(s, kt, n, qrow, lane);
+        f16x8 p[T::NB][2];
+        softmax_any<T, decltype(first)::value>(s, scale_log2, m_run, l_run, oacc, p);
+        pv_tile<T>(vbuf(hc, b), fr, p, oacc);
+    };
+    // wave-uniform branch; every part passes the same number of barriers. n_steps >= 1; step 0
+    // (each part's first tile) is peeled off.
+    with_part([&](auto hc) {
+        using Later = std::false_type;
+        step(0, hc, I0{}, std::true_type{});
+        int j = 1;
+        for (; j + 2 <= n_steps; j += 2) {
+            step(j, hc, I1{}, Later{});
+            step(j + 1, hc, I0{}, Later{});
+        }
+        if (j < n_steps) step(j, hc, I1{}, Later{});
+    });
+
+    // Merge: part 1 writes (m, l) to its buffer k10 and then O, one 32-column block at a time, to
+    // its buffer v10; part 0 merges. Lanes write 8 and 16 bytes at consecutive addresses (O as
+    // four 16-byte pieces per block, piece-major), which keeps every access free of bank conflicts.
+    float l_tot = sum_xor32(l_run);
+    const int slot = wq * 64 + lane;
+    wait_vmem();
+    __syncthreads();  // every wave is done with the tile buffers
+    f32x2* const ml = reinterpret_cast<f32x2*>(k10);
+    f32x4* const ob = reinterpret_cast<f32x4*>(v10);
+    if (part == 1) ml[slot] = f32x2{m_run, l_tot};
+    __syncthreads();
+    float wa = 1.0F, wb = 0.0F;
+    if (part == 0) {
+        const f32x2 mb_lb = ml[slot];
+        const float mb = mb_lb[0];
+        const float m_new = fmaxf(m_run, mb);
+        // a part that saw no key has m = -inf and weighs 0; both -inf only for rows >= n
+        wa = m_run == -INFINITY ? 0.0F : exp2_fast(m_run - m_new);
+        wb = mb == -INFINITY ? 0.0F : exp2_fast(mb - m_new);
+        l_tot = l_tot * wa + mb_lb[1] * wb;
+        m_run = m_new;
+    }
+#pragma unroll
+    for (int db = 0; db < T::DB; ++db) {
+        if (part == 1) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+                ob[r * T::NW * 64 + slot] = f32x4{oacc[db][4 * r], oacc[db][4 * r + 1],
+                                                  oacc[db][4 * r + 2], oacc[db][4 * r + 3]};
+        }
+        __syncthreads();
+        if (part == 0) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const f32x4 x = ob[r * T::NW * 64 + slot];
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    oacc[db][4 * r + i] = oacc[db][4 * r + i] * wa + x[i] * wb;
+            }
+        }
+        __syncthreads();
+    }
+    if (part == 0) {
+        store_o_tot<T>(o + head, lse ? lse + static_cast<size_t>(w.bh) * n : nullptr, qrow, n,
+                       lane, m_run, l_tot, oacc);
+    }
+}
+
+// ---- kernel, key-split schedule on 16x16x32 MFMAs (small grids) ---------------------------------
+// KS waves per 32 query rows (KS = 2, or 4 on grids of one workgroup per CU): wave w takes key
+// tiles part, part + KS, part + 2 KS, ... of the query block (part = w / NW) with its own running
+// max, row sum and O; the parts merge through LDS at the end. KS times the waves of the simple
+// schedule on the same grid, with no workspace.
+// What bounds it: a lone wave issues a VALU instruction about every 8 clocks (an exponential
+// every 16), so a step's softmax takes as long as its 32 MFMAs; 64 query rows per workgroup need
+// 16 KiB of K and V per part and step, and a CU takes 64 bytes of LDS DMA per clock; and a launch
+// has fixed costs (first loads 0.5-1.5 us, merge 0.5-1.5 us). Hence
+//   * fragment-order tiles (Frag16), row sums on the matrix cores (rowsum16): +1 to +3 % at d = 64;
+//   * KS = 2 (one or two workgroups per CU, waves that meet no partner on their SIMD): the step is
+//     pipelined inside the wave, S_{j+1} = K_{j+1} Q^T interleaved with the softmax of S_j, then
+//     O += P_j V_j while K_{j+2} is read. Two barriers per step (K_{j+1} read, V_j read), each
+//     followed by the refill of the buffer that it frees, one and a half steps before its use;
+//   * KS = 4 (two waves per SIMD): parts 0, 1 and 2, 3 run the ping-pong's two phases half a step
+//     apart (softmax and fragment reads; all MFMAs and the refill), so that one wave of a SIMD
+//     feeds the matrix pipe while the other is in its softmax (lockstep took 1.9 us a step of two
+//     tiles per SIMD at d = 128, this 1.6);
+//   * a merge of one exchange: every part writes the others' slices of O once and merges and
+//     stores its own slice (before, the parts merged pairwise, one 32-column block per barrier).
+// Measured against the 32x32x16 key split it replaces (MI355X, interleaved): d = 128 1x16x1000
+// 15.8 -> 13.6 us, 1x16x2000 43.3 -> 37.9, causal 1x16x2000 31.1 -> 26.4, 1x16x1000 15.2 -> 13.2,
+// 1x30x256 8.0 -> 7.3; d = 64 1x16x2000 24.3 -> 22.3, causal 17.8 -> 15.7, 1x4x900 9.5 -> 8.4.
+template <class T, bool CAUSAL, int KS>
+__global__ __launch_bounds__(T::THREADS) void flash_fwd_ksplit(
+    const f16* __restrict__ q, const f16* __restrict__ k, const f16* __restrict__ v,
+    f16* __restrict__ o, float* __restrict__ lse, int n, int bh_count, int n_qblocks,
+    float scale_log2, int negate_q, int /*tiles_per_split*/, float* /*o_part*/,
+    float* /*lse_part*/, unsigned /*launch_id*/, int /*group_heads*/) {
+    using G = M16<T>;
+    static_assert(KS == T::KS && (KS == 2 || KS == 4) && T::M16, "two or four key parts");
+    static_assert((T::D == 128 && T::BC == 32) || (T::D == 64 && T::BC == 64),
+                  "the 16x16x32 layouts are written for D=128, BC=32 and D=64, BC=64");
+    constexpr bool PHASES = KS == 4;  // two groups of waves, half a step apart
+    constexpr int TB = T::TILE_BYTES;
+    constexpr int IT = T::DMA_ITERS;  // requests per wave and tile
+    // A part's tile of step t in k_lds[t % 2] and v_lds[t % 2] (separate objects, so that the
+    // compiler sees that the refill of one cannot alias the reads of another).
+    __shared__ __attribute__((aligned(1024))) char k_lds0[KS * TB];
+    __shared__ __attribute__((aligned(1024))) char k_lds1[KS * TB];
+    __shared__ __attribute__((aligned(1024))) char v_lds0[KS * TB];
+    __shared__ __attribute__((aligned(1024))) char v_lds1[KS * TB];
+
+    const int lane = threadIdx.x & 63;
+    const int wave = wave_uniform(threadIdx.x >> 6);
+    const int part = wave / T::NW;  // key tiles part, part + KS, ...
+    const int wq = wave % T::NW;    // which 32 query rows
+    const int id = static_cast<int>(blockIdx.x);
+    const g::Work w = g::work_of_xcd(CAUSAL && KS == 2 ? g::two_round_turn(id, gridDim.x) : id,
+                                     bh_count, n_qblocks, CAUSAL);
+    const size_t head = static_cast<size_t>(w.bh) * n * T::D;
+    const f16* kh = k + head;
+    const f16* vh = v + head;
+    const int q0 = w.qb * T::BR;
+    const int qw = q0 + wq * 32;
+    const int n_tiles = g::num_kv_tiles(n, q0, T::BR, T::BC, CAUSAL);
+    const int n_steps = (n_tiles + KS - 1) / KS;
+    using I0 = std::integral_constant<int, 0>;
+    using I1 = std::integral_constant<int, 1>;
+    using I2 = std::integral_constant<int, 2>;
+    auto kbuf = [&](auto b) { return decltype(b)::value == 0 ? k_lds0 : k_lds1; };
+    auto vbuf = [&](auto b) { return decltype(b)::value == 0 ? v_lds0 : v_lds1; };
+
+    // Requests of a tile: the wave's IT pieces of 1 KiB. A tile past the part's last one has an
+    // empty buffer range (its requests read zeros), which keeps the steady steps free of branches
+    // and their vmcnt sequence fixed.
+    const TileDma<T, true> dma_k(wq, lane);
+    const TileDma<T> dma_v(wq, lane);
+    auto tile_at = [&](int j) { return KS * j + part; };
+    auto rsrc_of = [&](const f16* src, int j) {
+        const int t = tile_at(j);
+        const int rows = t < n_tiles ? n - t * T::BC : 0;
+        return make_rsrc(reinterpret_cast<const char*>(src) + static_cast<size_t>(t) * TB,
+                         static_cast<unsigned>(rows) * T::ROW_BYTES);
+    };
+    auto request = [&](__amdgpu_buffer_rsrc_t rsrc, int it, char* buf, const auto& dma) {
+        lds_dma16_buf(rsrc, dma.voff[it], buf + part * TB + (it * T::NW + wq) * 1024);
+    };
+    auto load = [&](const f16* src, int j, char* buf, const auto& dma) {
+        const auto rsrc = rsrc_of(src, j);
+#pragma unroll
+        for (int it = 0; it < IT; ++it) request(rsrc, it, buf, dma);
+    };
+    auto load_k = [&](int j, char* buf) { load(kh, j, buf, dma_k); };
+    auto load_v = [&](int j, char* buf) { load(vh, j, buf, dma_v); };
+    // The wave's LDS reads are complete, and of its requests all but those of the newest TILES
+    // tiles have landed; then the workgroup barrier.
+    auto fence = [&](auto tiles) {
+        constexpr int VM = decltype(tiles)::value * IT;
+        static_assert(VM < 16, "vmcnt field");
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_waitcnt(0x0070 | VM);
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+    };
+
+    const bool more = n_steps > 1;  // workgroup-uniform
+    load_k(0, k_lds0);
+    f16x8 qf[G::QB][G::DC];
+    load_q16<T>(q + head, qw, n, lane, 0, qf);
+    load_v(0, v_lds0);
+    if (more) load_k(1, k_lds1);
+    const int n_act = g::wave_active_tiles(n, qw, 32, T::BC, n_tiles, CAUSAL);
+    const int n_my = n_act > part ? (n_act - part + KS - 1) / KS : 0;  // steps with work
+    const Frag16<T> fr(lane, part * TB);
+    const unsigned qsign = negate_q != 0 ? 0x80008000U : 0U;
+#pragma unroll
+    for (int qb = 0; qb < G::QB; ++qb)
+#pragma unroll
+        for (int dc = 0; dc < G::DC; ++dc) qf[qb][dc] = xor_sign8(qf[qb][dc], qsign);
+
+    f32x4 oacc[G::DB][G::QB];
+#pragma unroll
+    for (int db = 0; db < G::DB; ++db)
+#pragma unroll
+        for (int qb = 0; qb < G::QB; ++qb) oacc[db][qb] = f32x4{};
+    float m_run[G::QB] = {-INFINITY, -INFINITY};
+    f32x4 l_run[G::QB] = {f32x4{}, f32x4{}};  // rowsum16
+    f32x4 s[G::KB][G::QB];
+    f16x8 kf[G::KB][G::DC];
+    f16x8 vf[G::KS][G::DB];
+    f16x8 p[G::QB][G::KS];
+    auto qk = [&](f32x4 (&sc)[G::KB][G::QB]) {
+#pragma unroll
+        for (int dc = 0; dc < G::DC; ++dc)
+#pragma unroll
+            for (int kb = 0; kb < G::KB; ++kb)
+#pragma unroll
+                for (int qb = 0; qb < G::QB; ++qb)
+                    sc[kb][qb] =
+                        mfma16(kf[kb][dc], qf[qb][dc], dc == 0 ? f32x4{} : sc[kb][qb]);
+    };
+    auto exact = [&](const f32x4 (&sc)[G::KB][G::QB], bool first) __attribute__((always_inline)) {
+        float alpha[G::QB];
+        bool rescale;
+        softmax16_tile_mx<T>(sc, scale_log2, m_run, l_run, alpha, rescale, p);
+        if (rescale && !first) rescale16<T>(oacc, alpha);
+    };
+
+    // S_0. A wave with further steps takes its running max from it (only a wave's last tile is
+    // ever masked), so that step 0 can run the optimistic softmax.
+    if (!more) {
+        fence(I1{});  // K_0 and Q have landed
+    } else {
+        fence(I2{});
+    }
+    if (n_my > 0) {
+        load_k16<T>(k_lds0, fr, kf);
+        qk(s);
+        if (n_my > 1) {
+#pragma unroll
+            for (int qb = 0; qb < G::QB; ++qb) {
+                float x = -INFINITY;
+#pragma unroll
+                for (int kb = 0; kb < G::KB; ++kb)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) x = fmaxf(x, s[kb][qb][r]);
+                m_run[qb] = max_xor32(max_xor16(x)) * scale_log2;
+            }
+        }
+    }
+    if (more) {
+        fence(I0{});  // V_0 and K_1; every wave has read K_0
+        load_k(2, k_lds0);
+        load_v(1, v_lds1);
+        if (!PHASES) load_k16<T>(k_lds1, fr, kf);
+    } else if constexpr (PHASES) {
+        fence(I0{});
+    }
+
+    int j = 0;
+    if constexpr (PHASES) {
+        // Step j (not the wave's last), B = j % 2. Softmax phase: K_{j+1} and V_j fragments, P_j.
+        // Matrix phase: S_{j+1}, O += P_j V_j and the refills K_{j+3}, V_{j+2} of the two buffers
+        // that every wave of the part has read by the barrier in between; K_{j+2} and V_{j+1},
+        // requested one step earlier, have landed by its end. Parts 2 and 3 run one phase behind.
+        if (part >= KS / 2) end_phase<false>();
+        auto step = [&](int jj, auto b) {
+            constexpr int B = decltype(b)::value;
+            using Other = std::integral_constant<int, 1 - B>;
+            load_k16<T>(kbuf(Other{}), fr, kf);
+            load_v16<T>(vbuf(b), fr, vf);
+            bool overflow;
+            softmax16_optimistic_mx<T>(s, scale_log2, m_run, l_run, overflow, p);
+            sched_reads_valu<8, T::D == 64 ? 48 : 24, 1, 16>();
+            end_phase<false>();
+            if (__builtin_expect(overflow, 0)) exact(s, false);
+            __builtin_amdgcn_s_setprio(1);
+            constexpr int NCH = G::KB * G::QB;  // QK chains
+            const auto rk = rsrc_of(kh, jj + 3);
+            const auto rv = rsrc_of(vh, jj + 2);
+#pragma unroll
+            for (int kb = 0; kb < G::KB; ++kb)
+#pragma unroll
+                for (int qb = 0; qb < G::QB; ++qb) s[kb][qb] = f32x4{};
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+                const int ch = i % NCH;
+                const int dc = i / NCH;
+                const int db = (i / G::QB) % G::DB;
+                const int qv = i % G::QB;
+                const int t = i / (G::QB * G::DB);
+                f32x4& sc = s[ch / G::QB][ch % G::QB];
+                sc = mfma16(kf[ch / G::QB][dc], qf[ch % G::QB][dc], sc);
+                oacc[db][qv] = mfma16(vf[t][db], p[qv][t], oacc[db][qv]);
+                __builtin_amdgcn_sched_barrier(0);  // keep the alternation, spread the requests
+                if (i % 2 == 1 && i < 2 * IT) {
+                    request(rk, i / 2, kbuf(Other{}), dma_k);
+                    request(rv, i / 2, vbuf(b), dma_v);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            }
+            __builtin_amdgcn_s_setprio(0);
+            fence(I2{});
+        };
+        for (; j + 2 < n_my; j += 2) {
+            step(j, I0{});
+            step(j + 1, I1{});
+        }
+        if (j + 1 < n_my) {
+            step(j, I0{});
+            ++j;
+        }
+    } else if (n_my > 1) {
+        // Step j (not the wave's last), B = j % 2: sc = S_j, kf = K_{j+1}; leaves S_{j+1} in sn and
+        // K_{j+2} in kf.
+        f32x4 s2[G::KB][G::QB];
+        auto step = [&](int jj, auto b, f32x4 (&sc)[G::KB][G::QB], f32x4 (&sn)[G::KB][G::QB]) {
+            constexpr int B = decltype(b)::value;
+            using Other = std::integral_constant<int, 1 - B>;
+            fence(I2{});  // V_j; every wave has read K_{j+1}
+            load_k(jj + 3, kbuf(Other{}));
+            load_v16<T>(vbuf(b), fr, vf);
+            bool overflow;
+            qk(sn);
+            softmax16_optimistic_mx<T>(sc, scale_log2, m_run, l_run, overflow, p);
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
+                __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+                __builtin_amdgcn_sched_group_barrier(0x402, T::D == 128 ? 7 : 14, 0);
+            }
+            if (__builtin_expect(overflow, 0)) exact(sc, false);
+            fence(I2{});  // K_{j+2}; every wave has read V_j
+            load_v(jj + 2, vbuf(b));
+            load_k16<T>(kbuf(b), fr, kf);
+            pv16<T>(vf, p, oacc);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
+                __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+                __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
+            }
+        };
+        for (; j + 2 < n_my; j += 2) {
+            step(j, I0{}, s, s2);
+            step(j + 1, I1{}, s2, s);
+        }
+        if (j + 1 < n_my) {
+            step(j, I0{}, s, s2);
+            ++j;
+#pragma unroll
+            for (int kb = 0; kb < G::KB; ++kb)
+#pragma unroll
+                for (int qb = 0; qb < G::QB; ++qb) s[kb][qb] = s2[kb][qb];
+        }
+    }
+    // The wave's last step (the only masked tile), then the steps in which only other waves of
+    // the workgroup have work: its share of the refills, in the steady steps' barrier order.
+    for (bool work = n_my > 0; j < n_steps; ++j, work = false) {
+        const bool refill = tile_at(j + 2) < n_tiles;  // K_{j+3} may be past the end (zeros)
+        char* const kb_j = j % 2 == 0 ? k_lds1 : k_lds0;
+        char* const vb_j = j % 2 == 0 ? v_lds0 : v_lds1;
+        if constexpr (!PHASES) {
+            fence(I0{});
+            if (refill) load_k(j + 3, kb_j);
+        }
+        if (work) {
+            load_v16<T>(vb_j, fr, vf);
+            const int kt = tile_at(j) * T::BC;
+            if (g::tile_needs_mask(n, kt, T::BC, qw, CAUSAL))
+                mask16_lim<T, CAUSAL>(s, kt, n, qw, lane);
+            bool overflow = true;
+            if (n_my > 1) softmax16_optimistic_mx<T>(s, scale_log2, m_run, l_run, overflow, p);
+            if (overflow) exact(s, n_my == 1);
+        }
+        if constexpr (PHASES) {
+            end_phase<false>();
+            if (refill) {
+                load_k(j + 3, kb_j);
+                load_v(j + 2, vb_j);
+            }
+            if (work) pv16<T>(vf, p, oacc);
+            if (refill) {
+                fence(I2{});
+            } else {
+                fence(I0{});
+            }
+        } else {
+            if (j + 1 < n_steps) fence(I0{});
+            if (refill) load_v(j + 2, vb_j);
+            if (work) pv16<T>(vf, p, oacc);
+        }
+    }
+    if (PHASES && part < KS / 2) end_phase<false>();
+
+    wait_vmem();  // (the requests past the last tile)
+    __syncthreads();
+    // Merge: every part hands each other part that part's slice of the features (SDB blocks) with
+    // its (m, l), and merges and stores its own slice. Part d's buffer xbuf[d] receives its slice
+    // from the others, 16 bytes per lane at consecutive addresses (no bank conflicts).
+    constexpr int SDB = G::DB / KS;
+    constexpr int WB = SDB * G::QB * 64;  // f32x4 per slice and wave
+    constexpr int ML_BYTES = KS * T::NW * G::QB * 64 * 8;
+    static_assert((KS - 1) * T::NW * WB * 16 + (KS == 4 ? ML_BYTES : 0) <= KS * TB &&
+                      ML_BYTES <= KS * TB,
+                  "the exchanged slices and (m, l) fit");
+    f32x4* const xbuf[4] = {reinterpret_cast<f32x4*>(k_lds0), reinterpret_cast<f32x4*>(k_lds1),
+                            reinterpret_cast<f32x4*>(v_lds0), reinterpret_cast<f32x4*>(v_lds1)};
+    f32x2* const ml = reinterpret_cast<f32x2*>(KS == 4 ? k_lds0 + 3 * T::NW * WB * 16 : v_lds0);
+    auto merge = [&](auto own) {
+        constexpr int P = decltype(own)::value;
+        float l_tot[G::QB];
+#pragma unroll
+        for (int qb = 0; qb < G::QB; ++qb) {
+            l_tot[qb] = l_run[qb][0];
+            ml[((P * T::NW + wq) * G::QB + qb) * 64 + lane] = f32x2{m_run[qb], l_tot[qb]};
+        }
+#pragma unroll
+        for (int d = 0; d < KS; ++d) {
+            if (d == P) continue;
+            f32x4* dst = xbuf[d] + ((P < d ? P : P - 1) * T::NW + wq) * WB + lane;
+#pragma unroll
+            for (int i = 0; i < SDB; ++i)
+#pragma unroll
+                for (int qb = 0; qb < G::QB; ++qb)
+                    dst[(i * G::QB + qb) * 64] = oacc[d * SDB + i][qb];
+        }
+        __syncthreads();
+        f32x2 x[KS][G::QB];
+        f32x4 y[KS][SDB][G::QB];
+#pragma unroll
+        for (int d = 0; d < KS; ++d)
+#pragma unroll
+            for (int qb = 0; qb < G::QB; ++qb)
+                x[d][qb] = d == P ? f32x2{m_run[qb], l_tot[qb]}
+                                  : ml[((d * T::NW + wq) * G::QB + qb) * 64 + lane];
+#pragma unroll
+        for (int d = 0; d < KS; ++d)
+#pragma unroll
+            for (int i = 0; i < SDB; ++i)
+#pragma unroll
+                for (int qb = 0; qb < G::QB; ++qb)
+                    y[d][i][qb] = d == P ? oacc[d * SDB + i][qb]
+                                         : xbuf[P][((d < P ? d : d - 1) * T::NW + wq) * WB + lane +
+                                                   (i * G::QB + qb) * 64];
+        f32x4 acc[SDB][G::QB];
+        float m_all[G::QB];
+        float l_all[G::QB];
+#pragma unroll
+        for (int qb = 0; qb < G::QB; ++qb) {
+            // a part that saw no key has l = 0 and weighs 0
+            float m = -INFINITY;
+#pragma unroll
+            for (int d = 0; d < KS; ++d) m = x[d][qb][1] > 0.0F ? fmaxf(m, x[d][qb][0]) : m;
+            float l = 0.0F;
+#pragma unroll
+            for (int d = 0; d < KS; ++d) {
+                const float wgt = x[d][qb][1] > 0.0F ? exp2_fast(x[d][qb][0] - m) : 0.0F;
+                l += wgt * x[d][qb][1];
+#pragma unroll
+                for (int i = 0; i < SDB; ++i)
+                    acc[i][qb] = d == 0 ? y[d][i][qb] * wgt : acc[i][qb] + y[d][i][qb] * wgt;
+            }
+            m_all[qb] = m;
+            l_all[qb] = l;
+            const float inv = l > 0.0F ? 1.0F / l : 0.0F;
+#pragma unroll
+            for (int i = 0; i < SDB; ++i) acc[i][qb] *= inv;
+        }
+        const int grp = lane >> 4;
+        f16* const oh = o + head + P * SDB * 16;
+#pragma unroll
+        for (int qb = 0; qb < G::QB; ++qb) {
+            const int qrow = qw + g::st16_query(lane, qb);
+            if constexpr (SDB >= 2) {
+                f16x8 out[SDB / 2];
+#pragma unroll
+                for (int e = 0; e < SDB / 2; ++e) {
+                    const f32x4& u = acc[2 * e][qb];
+                    const f32x4& t = acc[2 * e + 1][qb];
+                    out[e] = pair_swap16(pack4(u[0], u[1], u[2], u[3]), pack4(t[0], t[1], t[2], t[3]));
+                }
+                f16* dst = oh + static_cast<size_t>(qrow) * G::D + 4 * grp + 12 * (grp & 1);
+#pragma unroll
+                for (int e = 0; e < SDB / 2; ++e)
+                    if (qrow < n) *reinterpret_cast<f16x8*>(dst + 32 * e) = out[e];
+            } else if (qrow < n) {
+                const f32x4& u = acc[0][qb];
+                *reinterpret_cast<f16x4*>(oh + static_cast<size_t>(qrow) * G::D + 4 * grp) =
+                    pack4(u[0], u[1], u[2], u[3]);
+            }
+            if (P == 0 && lse != nullptr && lane < 16 && qrow < n)
+                lse[static_cast<size_t>(w.bh) * n + qrow] = row_lse2(m_all[qb], l_all[qb]) * kLn2;
+        }
+    };
+    if (part == 0) {
+        merge(I0{});
+    } else if (KS == 2 || part == 1) {
+        merge(I1{});
+    } else if (part == 2) {
+        merge(std::integral_constant<int, KS == 4 ? 2 : 0>{});
+    } else {
+        merge(std::integral_constant<int, KS == 4 ? 3 : 0>{});
+    }
+}
+
 // ---- tile table -------------------------------------------------------------------------------
 // Counterpart of the reference's per-(variant, d, causal) `using` lines
 // (csrc/kernels/flash_fwd.cu:597-612). On MI355X the best tile also depends on the sequence
@@ -2344,15 +2765,43 @@ __global__ __launch_bounds__(T::THREADS) void flash_fwd_simple16(
 #ifndef FA_OPT_D64_SMALL
 #define FA_OPT_D64_SMALL 64, 2, true, KSPLIT
 #endif
+// ... on 32x32x16 MFMAs (flash_fwd_ksplit<T, CAUSAL>) where a workgroup's fixed costs weigh most:
+//   * d = 64 up to FA_KS_SHORT_MAX_N keys: 1x4x384 5.55 us against 5.64 on 16x16x32, 1x4x256 4.71 /
+//     4.97, 1x30x128 4.05 / 4.31, but 1x17x385 6.50 / 6.24, 1x17x500 6.68 / 6.35 (up to 448 keys on
+//     the larger grids below: 1x62x420 9.12 / 9.15, 1x62x500 10.00 / 9.85);
+//   * causal grids of more than FA_KS_SHORT_BLOCKS query blocks of 64 rows up to FA_KS_SHORT_CAUSAL_
+//     MAX_N keys: d = 64 1x62x500 9.3 / 10.2, 1x62x700 14.7 / 15.4, 1x62x850 19.3 / 19.1; d = 128
+//     1x62x500 15.0 / 15.7, 1x62x700 21.7 / 23.4, 1x48x900 21.7 / 21.7 (with fewer blocks d = 64
+//     1x34x768 10.4 / 9.8, d = 128 1x40x700 14.9 / 13.1).
+#ifndef FA_OPT_D64_SMALL_SHORT
+#define FA_OPT_D64_SMALL_SHORT 64, 2, true, KSPLIT, false
+#endif
+#ifndef FA_OPT_D128_SMALL_SHORT
+#define FA_OPT_D128_SMALL_SHORT 32, 2, true, KSPLIT, false
+#endif
+#ifndef FA_KS_SHORT_MAX_N
+#define FA_KS_SHORT_MAX_N 384
+#endif
+#ifndef FA_KS_SHORT_BLOCKS
+#define FA_KS_SHORT_BLOCKS 400
+#endif
+#ifndef FA_KS_SHORT_CAUSAL_MAX_N
+#define FA_KS_SHORT_CAUSAL_MAX_N 800
+#endif
 #ifndef FA_OPT_D128_SMALL
 #define FA_OPT_D128_SMALL 32, 2, true, KSPLIT
 #endif
 // Grids of at most FA_TINY_GRID_WGS 64-row query blocks (one round of one workgroup per CU)
 // whose key loop has at least FA_TINY_MIN_TILES tiles: four waves per 32 query rows, each on
 // every fourth key tile (128 KiB of LDS, eight waves). Against the two-way split, interleaved on
-// one box: 1x8x2048 d=64 causal +12.7 %, 2x4x1500 d=128 causal +11.8 %, 2x8x1000 d=128 causal
-// +4.5 %, 1x16x1024 d=128 +1.7 %, 2x8x1000 d=64 causal (16 tiles) +1.9 %; with 8 tiles
-// (4x8x500 d=64) -7.7 %, with 4 (1x4x256 d=64) -13.8 %.
+// one box (32x32x16 key split): 1x8x2048 d=64 causal +12.7 %, 2x4x1500 d=128 causal +11.8 %,
+// 2x8x1000 d=128 causal +4.5 %, 1x16x1024 d=128 +1.7 %, 2x8x1000 d=64 causal (16 tiles) +1.9 %;
+// with 8 tiles (4x8x500 d=64) -7.7 %, with 4 (1x4x256 d=64) -13.8 %.
+// Causal grids of up to twice as many blocks take it from FA_TINY_CAUSAL_MIN_N_* keys: longest
+// first, the CUs that end a shorter block early take the short ones, and the longest block's
+// chain of steps is half as long. KSPLIT -> KSPLIT4: d = 128 1x8x4000 46.0 -> 42.3 us, 1x10x3000
+// 35.0 -> 32.7, 1x8x3500 38.9 -> 35.3, 1x16x2000 even, 1x16x1800 22.8 -> 24.6; d = 64 1x4x8192
+// 52.4 -> 47.1, 1x5x5000 32.6 -> 29.2, 1x8x3500 23.7 / 23.6, 1x16x2000 16.0 -> 18.4.
 #ifndef FA_OPT_D64_TINY
 #define FA_OPT_D64_TINY 64, 2, true, KSPLIT4
 #endif
@@ -2364,6 +2813,12 @@ __global__ __launch_bounds__(T::THREADS) void flash_fwd_simple16(
 #endif
 #ifndef FA_TINY_MIN_TILES
 #define FA_TINY_MIN_TILES 16
+#endif
+#ifndef FA_TINY_CAUSAL_MIN_N_D64
+#define FA_TINY_CAUSAL_MIN_N_D64 4096
+#endif
+#ifndef FA_TINY_CAUSAL_MIN_N_D128
+#define FA_TINY_CAUSAL_MIN_N_D128 2560
 #endif
 #ifndef FA_OPT_D64
 #define FA_OPT_D64 64, 8, true, SIMPLE16
@@ -2452,7 +2907,9 @@ struct Entry {
 };
 enum TileId : int {
     BASE_D64, BASE_D64_C, BASE_D128, BASE_D128_C,
-    OPT_D64_SMALL, OPT_D64_C_SMALL, OPT_D128_SMALL, OPT_D128_C_SMALL,
+    OPT_D64_SMALL, OPT_D64_C_SMALL, OPT_D64_SMALL_SHORT, OPT_D64_C_SMALL_SHORT,
+    OPT_D128_C_SMALL_SHORT,
+    OPT_D128_SMALL, OPT_D128_C_SMALL,
     OPT_D64_TINY, OPT_D64_C_TINY, OPT_D128_TINY, OPT_D128_C_TINY,
     OPT_D64, OPT_D64_ONE_ROUND, OPT_D64_C_SHORT, OPT_D64_C, OPT_D64_C_ROUND, OPT_D128_VSHORT,
     OPT_D128_SHORT, OPT_D128,
@@ -2465,6 +2922,9 @@ template <> struct Row<BASE_D128> : Entry<Tile<128, FA_BASE_D128>, false> {};
 template <> struct Row<BASE_D128_C> : Entry<Tile<128, FA_BASE_D128>, true> {};
 template <> struct Row<OPT_D64_SMALL> : Entry<Tile<64, FA_OPT_D64_SMALL>, false> {};
 template <> struct Row<OPT_D64_C_SMALL> : Entry<Tile<64, FA_OPT_D64_SMALL>, true> {};
+template <> struct Row<OPT_D64_SMALL_SHORT> : Entry<Tile<64, FA_OPT_D64_SMALL_SHORT>, false> {};
+template <> struct Row<OPT_D64_C_SMALL_SHORT> : Entry<Tile<64, FA_OPT_D64_SMALL_SHORT>, true> {};
+template <> struct Row<OPT_D128_C_SMALL_SHORT> : Entry<Tile<128, FA_OPT_D128_SMALL_SHORT>, true> {};
 template <> struct Row<OPT_D128_SMALL> : Entry<Tile<128, FA_OPT_D128_SMALL>, false> {};
 template <> struct Row<OPT_D128_C_SMALL> : Entry<Tile<128, FA_OPT_D128_SMALL>, true> {};
 template <> struct Row<OPT_D64_TINY> : Entry<Tile<64, FA_OPT_D64_TINY>, false> {};
@@ -2492,11 +2952,19 @@ TileId tile_id(int head_dim, bool causal, int variant, int n, int64_t bh) {
     if (bh * ((static_cast<int64_t>(n) + 255) / 256) < FA_SMALL_GRID_WGS) {
         const int bc =
             head_dim == 64 ? Tile<64, FA_OPT_D64_TINY>::BC : Tile<128, FA_OPT_D128_TINY>::BC;
-        if (bh * ((static_cast<int64_t>(n) + 63) / 64) <= FA_TINY_GRID_WGS &&
+        const int64_t blocks = bh * ((static_cast<int64_t>(n) + 63) / 64);
+        const int turn_n = head_dim == 64 ? FA_TINY_CAUSAL_MIN_N_D64 : FA_TINY_CAUSAL_MIN_N_D128;
+        const int64_t most = FA_TINY_GRID_WGS * (causal && n >= turn_n ? 2 : 1);
+        if (blocks <= most &&
             (n + bc - 1) / bc >= FA_TINY_MIN_TILES) {
             if (head_dim == 64) return causal ? OPT_D64_C_TINY : OPT_D64_TINY;
             return causal ? OPT_D128_C_TINY : OPT_D128_TINY;
         }
+        const bool many = blocks > FA_KS_SHORT_BLOCKS;
+        const bool short_causal = causal && many && n <= FA_KS_SHORT_CAUSAL_MAX_N;
+        if (head_dim == 64 && (short_causal || n <= (many ? 448 : FA_KS_SHORT_MAX_N)))
+            return causal ? OPT_D64_C_SMALL_SHORT : OPT_D64_SMALL_SHORT;
+        if (short_causal) return OPT_D128_C_SMALL_SHORT;
         if (head_dim == 64) return causal ? OPT_D64_C_SMALL : OPT_D64_SMALL;
         return causal ? OPT_D128_C_SMALL : OPT_D128_SMALL;
     }
@@ -2531,6 +2999,9 @@ decltype(auto) with_row(TileId id, F&& f) {
         case BASE_D128_C: return f(Row<BASE_D128_C>{});
         case OPT_D64_SMALL: return f(Row<OPT_D64_SMALL>{});
         case OPT_D64_C_SMALL: return f(Row<OPT_D64_C_SMALL>{});
+        case OPT_D64_SMALL_SHORT: return f(Row<OPT_D64_SMALL_SHORT>{});
+        case OPT_D64_C_SMALL_SHORT: return f(Row<OPT_D64_C_SMALL_SHORT>{});
+        case OPT_D128_C_SMALL_SHORT: return f(Row<OPT_D128_C_SMALL_SHORT>{});
         case OPT_D128_SMALL: return f(Row<OPT_D128_SMALL>{});
         case OPT_D128_C_SMALL: return f(Row<OPT_D128_C_SMALL>{});
         case OPT_D64_TINY: return f(Row<OPT_D64_TINY>{});
@@ -2638,7 +3109,11 @@ int launch(const fa_params& p, float* lse, hipStream_t stream, Scale sc, int n_s
             }
         }
     } else if constexpr (T::SCHED == KSPLIT || T::SCHED == KSPLIT4) {
-        fn = reinterpret_cast<const void*>(&flash_fwd_ksplit<T, CAUSAL>);
+        if constexpr (T::M16) {
+            fn = reinterpret_cast<const void*>(&flash_fwd_ksplit<T, CAUSAL, T::KS>);
+        } else {
+            fn = reinterpret_cast<const void*>(&flash_fwd_ksplit<T, CAUSAL>);
+        }
     } else if constexpr (T::SCHED == SIMPLE16) {
         fn = reinterpret_cast<const void*>(&flash_fwd_simple16<T, CAUSAL>);
     } else {

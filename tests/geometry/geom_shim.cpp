@@ -36,6 +36,7 @@ int geom_fo_kslot_row(int slot, int d) { return g::fo_kslot_row(slot, d); }
 int geom_fo_kslot_chunk(int slot, int d) { return g::fo_kslot_chunk(slot, d); }
 int geom_fo_vslot_row(int slot, int d) { return g::fo_vslot_row(slot, d); }
 int geom_fo_vslot_chunk(int slot, int d) { return g::fo_vslot_chunk(slot, d); }
+int geom_two_round_turn(int block_id, int total) { return g::two_round_turn(block_id, total); }
 int geom_tile_offset_m16(int row, int chunk, int d) { return g::tile_offset_m16(row, chunk, d); }
 int geom_st16_key(int lane, int kb, int r) { return g::st16_key(lane, kb, r); }
 int geom_st16_query(int lane, int qb) { return g::st16_query(lane, qb); }
