@@ -629,16 +629,41 @@ __global__ __launch_bounds__(256) void flash_fwd_combine(
         splits = min(n_splits, g::ceil_div(g::ceil_div(kv_end, block_k), tiles_per_split));
     }
     const size_t plane = static_cast<size_t>(bh_count) * n;  // rows per split
+    // Four splits at a time, so that their loads are in flight together (a split past the last one
+    // repeats the last and is left out): one after the other, the splits' load latencies bound
+    // it. Measured on MI355X with the sums in the same order: 12.0 -> 10.0 us at causal d = 64
+    // 1x1x16384, 7.5 -> 6.4 us at causal d = 128 1x2x4096, 7.5 -> 7.0 us at d = 128 1x1x16384
+    // (14.6 -> 15.1 us at causal d = 128 1x2x16384, whose pair of launches takes the same time).
+    constexpr int U = 4;
     float m = -INFINITY;
-    for (int s = 0; s < splits; ++s) m = fmaxf(m, lse_part[s * plane + row]);
+    for (int s0 = 0; s0 < splits; s0 += U) {
+        float x[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) x[u] = lse_part[min(s0 + u, splits - 1) * plane + row];
+#pragma unroll
+        for (int u = 0; u < U; ++u) m = fmaxf(m, x[u]);
+    }
     float wsum = 0.0F;
     f32x4 acc0{}, acc1{};
-    for (int s = 0; s < splits; ++s) {
-        const float wgt = exp2_fast(lse_part[s * plane + row] - m);
-        const float* src = o_part + (s * plane + row) * D + c;
-        wsum += wgt;
-        acc0 += wgt * *reinterpret_cast<const f32x4*>(src);
-        acc1 += wgt * *reinterpret_cast<const f32x4*>(src + 4);
+    for (int s0 = 0; s0 < splits; s0 += U) {
+        float x[U];
+        f32x4 y0[U], y1[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const size_t part = min(s0 + u, splits - 1) * plane + row;
+            x[u] = lse_part[part];
+            const float* src = o_part + part * D + c;
+            y0[u] = *reinterpret_cast<const f32x4*>(src);
+            y1[u] = *reinterpret_cast<const f32x4*>(src + 4);
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            if (s0 + u >= splits) break;
+            const float wgt = exp2_fast(x[u] - m);
+            wsum += wgt;
+            acc0 += wgt * y0[u];
+            acc1 += wgt * y1[u];
+        }
     }
     const float inv = 1.0F / wsum;  // >= 1: the split holding the row's max weighs 1
     *reinterpret_cast<f16x8*>(o + row * D + c) =
