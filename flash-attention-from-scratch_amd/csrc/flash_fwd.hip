@@ -3313,6 +3313,57 @@ bool splitkv_preferred(const fa_params& p) {
     return split_plan(p, 0).n_splits >= 2;
 }
 
+// Whether an automatic split (num_splits 0) runs as one launch of its row's key-split workgroups,
+// which share out a block's keys over their own waves and merge in LDS, instead of the partial
+// pass and its merge. Only below FA_SMALL_GRID_WGS blocks of 256 rows and from FA_SPLITKV_MIN_N
+// keys, where both were measured on MI355X (interleaved, both sides over 220 shapes; pair -> one
+// launch):
+//  - causal: the longest block bounds the one launch, so it needs at least two heads and 192
+//    blocks of 64 rows. d = 128 1x2x16384 160.9 -> 137.5 us, 1x4x8192 93.9 -> 73.5, 1x8x4096
+//    61.8 -> 41.9, 1x12x4096 81.1 -> 58.2, 1x3x4096 34.6 -> 30.8; d = 64 1x2x16384 95.7 -> 79.4.
+//    Outside: 1x1x16384 93.5 -> 103.5, 1x2x6000 (188 blocks) 38.5 -> 41.2, 1x1x8192 38.9 ->
+//    53.5, and past two rounds of long rows 1x3x20000 306 -> 315.
+//  - not causal: the pair's partial tile does more per read, so from FA_ONE_LAUNCH_MAX_N keys it
+//    wins (d = 128 1x1x32768 440 -> 519, 1x2x16384 230 -> 259, d = 64 1x2x16384 138 -> 148);
+//    below, its fixed part and its half-empty rounds cost more: d = 64 1x4x4096 37.5 -> 21.4,
+//    1x3x5000 49.4 -> 25.2, 1x4x6000 79.4 -> 50.3, 1x3x12000 189 -> 156; d = 128 1x3x5000 74.0
+//    -> 41.8, 1x6x5000 104.7 -> 81.2, 1x2x7000 91.1 -> 53.8, 1x3x8192 151 -> 115. It keeps the
+//    grids that fill its rounds (d = 128 1x1x8192 45.4 -> 54.1, 1x4x8192 124.5 -> 132.7; d = 64
+//    1x3x7000 49.1 -> 56.5) unless the one launch fills its own up to FA_ONE_LAUNCH_FULL_N_*
+//    keys (d = 64 1x2x8192 50.5 -> 39.3, 1x4x8192 78.8 -> 75.8; d = 128 1x4x4096 46.4 -> 36.8),
+//    grids past three rounds of 64-row blocks (d = 128 1x10x5000 145 -> 149; d = 64 1x7x8192
+//    138.5 -> 142.4, but 1x14x4096 81.1 -> 74.1), and very small ones at d = 128 (1x1x5000 32.1
+//    -> 36.1).
+#ifndef FA_ONE_LAUNCH_MAX_N
+#define FA_ONE_LAUNCH_MAX_N 12288
+#endif
+#ifndef FA_ONE_LAUNCH_FULL_N_D64
+#define FA_ONE_LAUNCH_FULL_N_D64 8192
+#endif
+#ifndef FA_ONE_LAUNCH_FULL_N_D128
+#define FA_ONE_LAUNCH_FULL_N_D128 6144
+#endif
+bool split_in_one_launch(const fa_params& p, const SplitPlan& sp) {
+    if (p.variant == FA_VARIANT_BASELINE || p.seqlen < FA_SPLITKV_MIN_N) return false;
+    const int64_t bh = static_cast<int64_t>(p.batch) * p.heads;
+    if (bh * ((static_cast<int64_t>(p.seqlen) + 255) / 256) >= FA_SMALL_GRID_WGS) return false;
+    const int64_t blocks = bh * ((static_cast<int64_t>(p.seqlen) + 63) / 64);
+    if (p.causal) {
+        return bh >= 2 && blocks >= 192 &&
+               (p.head_dim == 64 || blocks <= 2 * g::kCus || p.seqlen <= 16384);
+    }
+    if (p.seqlen > FA_ONE_LAUNCH_MAX_N) return false;
+    if (p.head_dim == 128 && blocks < 90) return false;
+    if (blocks > 3 * g::kCus && (p.head_dim == 128 || p.seqlen > 5120)) return false;
+    const auto fills = [](int64_t wgs) {  // no round of one workgroup per CU under 15/16 full
+        const int64_t last = wgs % g::kCus;
+        return last == 0 || 16 * last > 15 * g::kCus;
+    };
+    if (!fills(bh * g::ceil_div(p.seqlen, sp.block_q) * sp.n_splits)) return true;
+    return fills(blocks) && p.seqlen <= (p.head_dim == 64 ? FA_ONE_LAUNCH_FULL_N_D64
+                                                          : FA_ONE_LAUNCH_FULL_N_D128);
+}
+
 // Non-causal head split for grids whose last round of ping-pong workgroups (one per CU) is
 // mostly empty: the first `heads` (b, h) heads run as one launch whose items fill whole rounds,
 // the rest through the split-KV pair, whose key ranges fill the CUs. Returns that head count, or
@@ -3586,8 +3637,9 @@ static int splitkv_checks(const fa_params* params, float* lse, int32_t num_split
     return FA_OK;
 }
 
-static int splitkv_run(const fa_params& p, float* lse, const fa::SplitPlan& sp, void* workspace,
-                       void* stream) {
+static int splitkv_run(const fa_params& p, float* lse, int32_t num_splits,
+                       const fa::SplitPlan& sp, void* workspace, void* stream) {
+    if (num_splits == 0 && fa::split_in_one_launch(p, sp)) return run(p, lse, stream);
     const fa::Scale sc = fa::scale_of(p.softmax_scale);
     auto s = static_cast<hipStream_t>(stream);
     return fa::with_split_row(p, [&](auto row) {
@@ -3608,7 +3660,7 @@ int fa_flash_fwd_splitkv(const fa_params* params, float* lse, int32_t num_splits
         return fa::fail(FA_EINVAL, "flash_fwd_splitkv: workspace too small: need " +
                                        std::to_string(sp.workspace_bytes) + " bytes");
     }
-    return splitkv_run(*params, lse, sp, workspace, stream);
+    return splitkv_run(*params, lse, num_splits, sp, workspace, stream);
 }
 
 int fa_flash_fwd_splitkv_static(const fa_params* params, float* lse, int32_t num_splits,
@@ -3628,7 +3680,7 @@ int fa_flash_fwd_splitkv_static(const fa_params* params, float* lse, int32_t num
     void* ws = nullptr;
     const int src = fa::static_scratch(&ws);
     if (src != FA_OK) return src;
-    return splitkv_run(*params, lse, sp, ws, stream);
+    return splitkv_run(*params, lse, num_splits, sp, ws, stream);
 }
 
 }  // extern "C"

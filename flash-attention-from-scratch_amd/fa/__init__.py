@@ -76,7 +76,8 @@ def forward_splitkv(
 ) -> tuple[torch.Tensor, torch.Tensor]:
     """(O, LSE) computed split-KV: every query block's keys are cut into ranges processed by
     separate workgroups and merged by their LSEs. For grids too small to fill the GPU (few
-    heads, long sequences). num_splits = 0 picks the ranges automatically. Matches `forward`
+    heads, long sequences). num_splits = 0 picks the ranges automatically, or one launch whose
+    workgroups split the keys over their own waves where that is faster. Matches `forward`
     within fp32 rounding of the merge. Not in the reference package."""
     return _C.forward_splitkv(q, k, v, causal, softmax_scale, num_splits)
 

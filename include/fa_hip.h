@@ -91,8 +91,11 @@ int fa_flash_fwd_lse(const fa_params* params, float* lse, void* stream);
  * 256 to 1024 workgroups with work, by head_dim and causal), and whether the split path is the
  * faster one for these params; host-only. fa_flash_fwd_splitkv runs it: lse may be NULL;
  * workspace must be 16-byte aligned and hold at least workspace_bytes of the plan for the same
- * params and num_splits. Two launches on `stream`; allocates nothing. The variant field is
- * checked but every variant runs the same split tile. */
+ * params and num_splits. Two launches on `stream`, or one with num_splits 0 where a single launch
+ * whose workgroups split the keys over their own waves is the faster way to share them out (the
+ * plan and the checks are the same, the workspace is then left alone, and the results are
+ * fa_flash_fwd_lse's); allocates nothing. The variant field is checked; every variant runs the
+ * same split tile, and the baseline always the two launches. */
 typedef struct fa_splitkv_info {
     int32_t num_splits;       /* key ranges per query block (ranges past a causal block's last
                                  key tile are skipped)                                        */
@@ -106,7 +109,8 @@ typedef struct fa_splitkv_info {
                                  N >= 16384; or a causal grid of 256 to 288 query blocks of
                                  256 rows, N >= 8192, where the automatic plan takes two
                                  ranges at D = 128), else 0; independent of num_splits. The PyTorch
-                                 binding's forward takes the split path exactly when it is 1. */
+                                 binding's forward takes the split path exactly when it is 1
+                                 (which may run it as one launch, above). */
     int32_t reserved;         /* 0                                                            */
 } fa_splitkv_info;
 int fa_splitkv_plan(const fa_params* params, int32_t num_splits, fa_splitkv_info* out);

@@ -4,6 +4,7 @@ Lengths around a key tile, a step of two or four tiles, the switch to the 32x32x
 the four-way split's causal extension; inputs that leave the optimistic softmax (a row max that
 jumps far past 2^16 in a later step, a part whose keys all lie far below the others', so that its
 merge weight underflows); scales 0, negative and large; O and the LSE against the fp32 oracle.
+The automatic splits that run as one launch of it, on both sides of their rule.
 CPU: the order of the two-round causal grids is a permutation that ends with the longest blocks'
 partners.
 """
@@ -86,6 +87,54 @@ def test_softmax_paths_and_merge(d, n, causal, kind):
         level[torch.arange(n) // tile % 2 == 1] = -200.0
     k[..., 0] = (level * 0.6931 * d ** 0.5 / 4.0).half()
     _check(q, k, v, causal)
+
+
+# (B, H, N, d, causal, one): automatic splits on both sides of the rule that runs them as one launch
+ONE_LAUNCH = [(1, 3, 4096, 128, True, True), (1, 2, 6000, 128, True, False),
+              (2, 1, 8192, 128, True, True), (1, 1, 16384, 128, True, False),
+              (1, 2, 16384, 64, True, True), (1, 3, 4095, 64, True, False),
+              (1, 6, 5000, 64, True, True), (1, 3, 5000, 64, False, True),
+              (1, 3, 7000, 64, False, False), (1, 4, 8192, 64, False, True),
+              (1, 1, 12289, 64, False, False), (1, 13, 4500, 64, False, True),
+              (1, 1, 5000, 128, False, False), (1, 2, 7000, 128, False, True),
+              (1, 1, 8192, 128, False, False), (1, 10, 5000, 128, False, False)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("b,h,n,d,causal,one", ONE_LAUNCH)
+def test_automatic_split_in_one_launch(b, h, n, d, causal, one):
+    """num_splits = 0 against the single launch (the same bits where it is one launch), the
+    general pair with three key ranges (the forward's tolerance), the static entry point (the
+    same bits) and selected rows in fp64."""
+    import fa
+    from fa import native
+
+    print(f"case one launch B={b} H={h} N={n} d={d} causal={causal}", flush=True)
+    q, k, v = _qkv(b, h, n, d, seed=n + 7 * h)
+    qc, kc, vc = q.cuda(), k.cuda(), v.cuda()
+    o, lse = fa.forward_splitkv(qc, kc, vc, causal=causal)
+    o1, lse1 = torch.empty_like(o), torch.empty_like(lse)
+    p = native.make_params(qc.data_ptr(), kc.data_ptr(), vc.data_ptr(), o1.data_ptr(), b, h, n, d,
+                           d ** -0.5, causal, "opt")
+    stream = torch.cuda.current_stream().cuda_stream
+    rc, msg = native.flash_fwd_lse(p, lse1.data_ptr(), stream)
+    assert rc == native.FA_OK, msg
+    torch.cuda.synchronize()
+    same = torch.equal(o, o1) and torch.equal(lse, lse1)
+    assert same == one
+    if native.splitkv_plan(p, 0)["workspace_bytes"] <= 64 << 20:
+        rc, msg = native.flash_fwd_splitkv_static(p, lse1.data_ptr(), 0, stream)
+        assert rc == native.FA_OK, msg
+        torch.cuda.synchronize()
+        assert torch.equal(o, o1) and torch.equal(lse, lse1)
+    o2, lse2 = fa.forward_splitkv(qc, kc, vc, causal=causal, num_splits=3)
+    torch.testing.assert_close(o, o2, atol=ATOL, rtol=RTOL)
+    torch.testing.assert_close(lse, lse2, atol=2e-3, rtol=0)
+    rows = [0, 1, 63, 64, n // 2, n - 1]
+    for bh in {0, b * h - 1}:
+        got = o.view(b * h, n, d)[bh, rows].cpu().double()
+        want = torch.as_tensor(orc.attention_fp64_rows(q, k, v, causal, bh, rows))
+        torch.testing.assert_close(got, want, atol=ATOL, rtol=RTOL)
 
 
 @pytest.mark.parametrize("total", [1, 256, 257, 288, 400, 511, 512, 513, 1000])
